@@ -14,6 +14,28 @@ def hb(bridge):
     return bridge
 
 
+def test_pack_tables_prompt_rows(hb):
+    """Rows longer than the workgroup beside empty and one-token rows, first and last too."""
+    from hip_bridge import DeviceBuffer
+
+    rng = np.random.default_rng(12)
+    row_tokens = np.array([0, 1, 2500, 0, 0, 1023, 1, 1025, 0], np.int32)
+    rows, max_pages, page = len(row_tokens), 200, 16
+    positions = rng.integers(0, max_pages * page - 2500, rows).astype(np.int32)
+    bt = rng.permutation(rows * max_pages).reshape(rows, max_pages).astype(np.int32)
+    n = int(row_tokens.sum())
+    d = [DeviceBuffer.from_array(a) for a in (row_tokens, positions, bt)]
+    out = {k: DeviceBuffer(4 * m) for k, m in (("cu_seqlens", rows + 1), ("token_row", n), ("token_pos", n),
+                                              ("kv_slot", n), ("context", rows), ("status", 1))}
+    print("case: pack prompt rows", flush=True)
+    hb.pack_tables(d[0], d[1], d[2], max_pages, rows, page, *out.values())
+    hb.synchronize()
+    want = oracle.pack_tables(row_tokens, positions, bt, page)
+    assert out["status"].download(np.int32, 1)[0] == 0
+    for k in ("cu_seqlens", "token_row", "token_pos", "kv_slot", "context"):
+        assert np.array_equal(out[k].download(np.int32, len(want[k])), want[k]), k
+
+
 # tokens around the 16-token span and the 64-token span group; histories in the
 # first span's rows, across its end, in a later span, and past the row's tokens
 @pytest.mark.parametrize("in_place", [True, False])
