@@ -123,10 +123,16 @@ extern "C" int hb_paged_attention(const void* q, const void* kcache, const void*
         work_o + attn_work_floats_o(rows, kv_heads, head_dim, max_tokens, group, max_context, split_len));
     AttnWork w{rows, max_tokens, rgs, splits, split_len, work_o, work_ml, plan};
     const hipStream_t s = as_stream(stream);
+    const bf16_t* const gate = static_cast<const bf16_t*>(qg);
+    const bool prefill = attn_prefill_rows(g, w, tokens, gate, ld_qg, static_cast<const bf16_t*>(out));
     attn_plan(cu_seqlens, context, g, w, s);
+    if (prefill)
+      attn_prefill(static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(kcache),
+                   static_cast<const bf16_t*>(vcache), block_table, max_pages, cu_seqlens, context, g, scale, w, gate,
+                   ld_qg, static_cast<bf16_t*>(out), s);
     paged_attention(static_cast<const bf16_t*>(q), static_cast<const bf16_t*>(kcache),
                     static_cast<const bf16_t*>(vcache), block_table, max_pages, cu_seqlens, context, g, scale, w, s);
-    attn_combine(w, token_row, cu_seqlens, context, static_cast<const bf16_t*>(qg), ld_qg, tokens, g,
+    attn_combine(w, token_row, cu_seqlens, context, gate, ld_qg, tokens, g,
                  static_cast<bf16_t*>(out), s);
   });
 }

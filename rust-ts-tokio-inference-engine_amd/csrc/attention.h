@@ -42,7 +42,35 @@ struct AttnWork {
   float* work_o;
   float* work_ml;
   int32_t* plan;
+  // rows of at least prefill_from tokens (0: none) are attn_prefill's: the plan
+  // lists no piece for them and the combine leaves them alone; prefill_only:
+  // every row is
+  int prefill_from = 0;
+  bool prefill_only = false;
 };
+// Rows of at least kPrefillRowTokens tokens in one launch without partials
+// (attn_prefill.hip), gate included: true when the step may have such rows and
+// the operands fit (head_dim 256, 8-byte aligned gate and output), with
+// w.prefill_from and w.prefill_only set; false, with nothing launched, when
+// every row is left to the split kernel. Which kernel computes a row depends
+// on the row alone.
+//
+// A lone row's q tiles are all that run beside each other, each walking the
+// row's keys at 34 ns a key, while the split kernel spreads them over the chip:
+// 0.095 ns per token and key, plus some 15 us more for its list and merge.
+// So few tokens over many keys stay with the split (us, split / one launch: 64
+// tokens over 564 keys 28 / 31, over 964 29 / 44; 200 over 2,200 76 / 82; 256
+// over 6,256 177 / 213; 500 over 5,500 293 / 189; 500 over 500 83 / 30).
+constexpr int kPrefillRowTokens = 64;
+template <class I>
+__host__ __device__ inline bool attn_prefill_row(I tokens, I context, int from) {
+  return from && tokens >= from && (tokens >= 6 * from || context <= 8 * tokens);
+}
+bool attn_prefill_rows(const AttnGeom& g, AttnWork& w, int tokens, const bf16_t* qg, int ld_qg, const bf16_t* out);
+void attn_prefill(const bf16_t* q, const bf16_t* kcache, const bf16_t* vcache, const int32_t* block_table,
+                  int max_pages, const int32_t* cu_seqlens, const int32_t* context, const AttnGeom& g, float scale,
+                  const AttnWork& w, const bf16_t* qg, int ld_qg, bf16_t* out, hipStream_t stream);
+
 size_t attn_work_floats_o(int rows, int kv_heads, int head_dim, int max_tokens, int group, int max_context,
                           int split_len);
 size_t attn_plan_ints(int rows, int kv_heads, int row_groups, int splits);

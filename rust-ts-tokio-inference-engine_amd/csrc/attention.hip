@@ -178,10 +178,12 @@ struct RowPieces {
 };
 
 __device__ inline RowPieces row_pieces(const int32_t* __restrict__ cu_seqlens, const int32_t* __restrict__ context,
-                                       int r, int group, int row_groups, int splits, int split_len) {
+                                       int r, int group, int row_groups, int splits, int split_len,
+                                       int prefill_from) {
   RowPieces p{0, 0, 0};
-  const int ctx = context[r];
-  p.groups = min((cu_seqlens[r + 1] - cu_seqlens[r]) * group + 15, 16 * row_groups) / 16;
+  const int ctx = context[r], T = cu_seqlens[r + 1] - cu_seqlens[r];
+  if (attn_prefill_row(T, ctx, prefill_from)) return p;
+  p.groups = min(T * group + 15, 16 * row_groups) / 16;
   if (p.groups == 0 || ctx <= 0) return RowPieces{0, 0, 0};
   p.whole = min(ctx / split_len, splits);
   p.tail = p.whole < splits ? ctx % split_len : 0;
@@ -194,7 +196,8 @@ constexpr int kPlanBuckets = 32 * kMaxPieceSteps;  // short-piece lengths 1..spl
 __global__ __launch_bounds__(kPlanThreads) void attn_plan_kernel(const int32_t* __restrict__ cu_seqlens,
                                                                  const int32_t* __restrict__ context, int rows,
                                                                  int group, int row_groups, int splits, int split_len,
-                                                                 int Hkv, int32_t* __restrict__ plan) {
+                                                                 int Hkv, int prefill_from,
+                                                                 int32_t* __restrict__ plan) {
   __shared__ int sc[kPlanThreads];
   __shared__ int row_off[kPlanMaxRows + 1];  // first list slot of each row's whole pieces
   __shared__ short row_groups_s[kPlanMaxRows], row_tail[kPlanMaxRows];
@@ -207,7 +210,7 @@ __global__ __launch_bounds__(kPlanThreads) void attn_plan_kernel(const int32_t* 
     const int r = base + tid;
     RowPieces p{0, 0, 0};
     if (r < rows) {
-      p = row_pieces(cu_seqlens, context, r, group, row_groups, splits, split_len);
+      p = row_pieces(cu_seqlens, context, r, group, row_groups, splits, split_len, prefill_from);
       row_groups_s[r] = short(p.groups);
       row_tail[r] = short(p.tail);
       if (p.tail > 0) atomicAdd(&bucket[p.tail], p.groups * Hkv);
@@ -479,10 +482,11 @@ __global__ __launch_bounds__(256) void attn_combine_kernel(const float* __restri
                                                            const int32_t* __restrict__ cu_seqlens,
                                                            const bf16_t* __restrict__ qg, int ld_qg, int Hq, int Hkv,
                                                            int D, int row_groups, int splits, int split_len,
-                                                           const int32_t* __restrict__ context,
+                                                           const int32_t* __restrict__ context, int prefill_from,
                                                            bf16_t* __restrict__ out) {
   const int h = blockIdx.x, i = blockIdx.y, d = threadIdx.x;
   const int r = token_row[i], t = i - cu_seqlens[r];
+  if (attn_prefill_row(cu_seqlens[r + 1] - cu_seqlens[r], context[r], prefill_from)) return;  // uniform: no partials
   const int group = Hq / Hkv, kh = h / group, pair = t * group + h % group;
   const int rg = pair / 16, col = pair % 16;
   const int ns = (context[r] + split_len - 1) / split_len;
@@ -568,8 +572,9 @@ void attn_plan(const int32_t* cu_seqlens, const int32_t* context, const AttnGeom
   require(w.rows > 0 && w.rows <= kPlanMaxRows && w.row_groups > 0 && w.row_groups < 32768 && w.splits > 0 &&
               w.split_len > 0 && w.split_len <= kPlanBuckets && w.plan,
           "attn_plan: invalid work geometry (at most 2048 rows, split_len <= 256)");
+  if (w.prefill_only) return;
   hipLaunchKernelGGL(attn_plan_kernel, dim3(1), dim3(kPlanThreads), 0, stream, cu_seqlens, context, w.rows,
-                     g.q_heads / g.kv_heads, w.row_groups, w.splits, w.split_len, g.kv_heads, w.plan);
+                     g.q_heads / g.kv_heads, w.row_groups, w.splits, w.split_len, g.kv_heads, w.prefill_from, w.plan);
   HB_CHECK(hipGetLastError());
 }
 
@@ -580,6 +585,7 @@ void paged_attention(const bf16_t* q, const bf16_t* kcache, const bf16_t* vcache
   require(w.split_len > 0 && w.split_len % 32 == 0 && w.split_len <= 32 * kMaxPieceSteps,
           "paged_attention: split_len must be a multiple of 32, at most 256");
   require(w.row_groups * 16 >= w.max_tokens * (g.q_heads / g.kv_heads), "paged_attention: row groups");
+  if (w.prefill_only) return;
   // persistent: one wave per SIMD (the kernel holds one wave's registers per
   // SIMD), never more waves than pieces could need
   static int slots = 0;
@@ -602,10 +608,10 @@ void attn_combine(const AttnWork& w, const int32_t* token_row, const int32_t* cu
                   const bf16_t* qg, int ld_qg, int tokens, const AttnGeom& g, bf16_t* out, hipStream_t stream) {
   require(w.splits <= kMaxCombineSplits && g.head_dim >= 64 && g.head_dim <= 256,
           "attn_combine: at most 1024 splits and a head_dim of 64..256");
-  if (tokens <= 0) return;
+  if (tokens <= 0 || w.prefill_only) return;
   launch_timed(attn_combine_kernel, dim3(g.q_heads, tokens), dim3(g.head_dim), 0, stream, w.work_o, w.work_ml,
                token_row, cu_seqlens, qg, ld_qg, g.q_heads, g.kv_heads, g.head_dim, w.row_groups, w.splits,
-               w.split_len, context, out);
+               w.split_len, context, w.prefill_from, out);
   HB_CHECK(hipGetLastError());
 }
 

@@ -617,6 +617,17 @@ void Engine::upload_tables(const StepRows& s) {
     const int group = g_.Hq / g_.Hkv;
     attn_work_ = AttnWork{B, max_t, (max_t * group + 15) / 16, (max_ctx + attn_split_ - 1) / attn_split_,
                           attn_split_, attn_wo_, attn_wml_, attn_plan_};
+    if (attn_prefill_rows(ag, attn_work_, T, proj_, g_.attn_in_rows(), aout_)) {  // the rows are known here
+      bool any = false, all = true;
+      for (int r = 0; r < B; ++r) {
+        const int t = s.row_tokens[r];
+        const bool on = attn_prefill_row(t, s.positions[r] + t, attn_work_.prefill_from);
+        any |= on;
+        all &= on || t == 0;
+      }
+      attn_work_.prefill_only = any && all;
+      if (!any) attn_work_.prefill_from = 0;
+    }
     attn_plan(d_cu_, d_ctx_, ag, attn_work_, stream_);
   }
 }
@@ -725,10 +736,14 @@ void Engine::layer_forward(const LayerW& w, int attn_index, int dn_index, int T,
     op_begin();
     require(attn_work_.rows == B && attn_work_.max_tokens >= max_t, "engine: attention piece list of another step");
     const bool sampled = probe_sample(2);
-    probe_begin(2, sampled, false);
+    const bool prefill = attn_work_.prefill_from > 0;
+    probe_begin(2, sampled, attn_work_.prefill_only);  // one launch, or from the first to the combine
+    if (prefill)
+      attn_prefill(q_, kc_[pool], vc_[pool], d_bt_rows_, max_pages_, d_cu_, d_ctx_, ag, 1.f / std::sqrt(float(g.D)),
+                   attn_work_, proj_, rows, aout_, stream_);
     paged_attention(q_, kc_[pool], vc_[pool], d_bt_rows_, max_pages_, d_cu_, d_ctx_, ag, 1.f / std::sqrt(float(g.D)),
                     attn_work_, stream_);
-    probe_last(2, sampled);
+    if (!attn_work_.prefill_only) probe_last(2, sampled);
     attn_combine(attn_work_, d_tok_row_, d_cu_, d_ctx_, proj_, rows, T, ag, aout_, stream_);
     // K and V of every context token, then q, gate and the output per packed token (bf16)
     probe_end(2, T, sampled, step_ctx_sum_ * g.Hkv * g.D * 2 * 2 + double(T) * g.Hq * g.D * 2 * 3);

@@ -3,6 +3,7 @@ import numpy as np
 import pytest
 
 import oracle
+from numerics import assert_bf16_close
 
 pytestmark = pytest.mark.gpu
 
@@ -76,3 +77,83 @@ def test_gdn_prep_spans_equal_the_row_walk(hb, heads, in_place):
                    + [d[5].download(np.uint16, win.shape)])
     for name, a, b in zip(("q", "k", "v", "decay", "beta", "window"), *got):
         assert np.array_equal(a, b), f"{name}: {int(np.sum(a != b))} values differ"
+
+
+# prompt rows beside decode rows, at the prompt kernel's edges: 64 tokens (its
+# least), 16-token blocks and 32-key tiles full and one over, keys before the
+# prompt, rows on both sides of the rule that leaves few tokens over many keys to
+# the splits, a row without keys, a lone row (no split launches), head groupings of
+# 1 and 8
+@pytest.mark.parametrize("T,ctx", [
+    ([64, 1, 63, 130, 4], [64, 500, 70, 333, 4]),
+    ([97, 80, 64], [97, 607, 32 * 5]),
+    ([64, 64, 390, 383], [512, 513, 3200, 3100]),
+    ([64, 2, 64], [0, 300, 65]),
+    ([129], [129]),
+    ([65], [1000]),
+])
+@pytest.mark.parametrize("hq,hkv", [(16, 2), (2, 2)])
+def test_paged_attention_prompt_rows(hb, T, ctx, hq, hkv):
+    from hip_bridge import DeviceBuffer
+
+    dim, page, split = 256, 16, 256
+    rng = np.random.default_rng(sum(T) + hq)
+    rows, tokens, most, width = len(T), sum(T), max(T), max(ctx)
+    max_pages = (width + page - 1) // page
+    bt = rng.permutation(rows * max_pages).reshape(rows, max_pages).astype(np.int32)
+    bits = lambda *shape, std=1.0: hb.quant.bf16_bits(rng.standard_normal(shape, dtype=np.float32) * np.float32(std))  # noqa: E731
+    kc, vc = bits(rows * max_pages, hkv, page, dim), bits(rows * max_pages, hkv, page, dim)
+    q, qg = bits(tokens, hq, dim, std=3.0), bits(tokens, hq, 2 * dim)
+    cu = np.concatenate([[0], np.cumsum(T)]).astype(np.int32)
+    full = np.maximum(ctx, T).astype(np.int32)  # the oracle's context of a row without keys, whose output is zeros
+    obt = bt if full.max() <= max_pages * page else np.tile(bt, 2)
+    val = hb.quant.bf16_value
+    want = oracle.paged_attention(val(q), val(kc), val(vc), obt, cu, full, 1 / 16, gate=val(qg)[:, :, dim:].copy())
+    for r in range(rows):
+        if ctx[r] == 0:
+            want[cu[r]:cu[r + 1]] = 0.0
+    up = DeviceBuffer.from_array
+    nwo = hb.attn_workspace_floats(rows, hkv, dim, most, hq // hkv, width, split)
+    dev = [up(a) for a in (q, kc, np.ascontiguousarray(vc.transpose(0, 1, 3, 2)), bt, cu, np.asarray(ctx, np.int32),
+                           np.repeat(np.arange(rows, dtype=np.int32), T), qg)]
+    wo, wml, out = DeviceBuffer(4 * nwo), DeviceBuffer(4 * nwo // dim * 2 + 256), DeviceBuffer(tokens * hq * dim * 2)
+    print(f"case: prompt attention T={T} ctx={ctx} heads {hq}/{hkv}", flush=True)
+    hb.paged_attention(dev[0], dev[1], dev[2], dev[3], max_pages, dev[4], dev[5], dev[6], dev[7], hq * 2 * dim, rows,
+                       tokens, most, width, hq, hkv, dim, 1 / 16, split, wo, wml, out)
+    hb.synchronize()
+    got = val(out.download(np.uint16, (tokens, hq, dim)))
+    for r in range(rows):  # each row by its own scale
+        sl = slice(cu[r], cu[r + 1])
+        if ctx[r] == 0:
+            assert not got[sl].any(), f"row {r} has no keys"
+        else:
+            assert_bf16_close(got[sl], want[sl], f"row {r}: {T[r]} tokens, context {ctx[r]}")
+
+
+def test_paged_attention_prompt_sink(hb):
+    """One key far above all later ones (by about 2^170 in weight): the later
+    keys' reference may not lift it out of range, and the rows see it alone."""
+    from hip_bridge import DeviceBuffer
+
+    dim, page, T, split = 256, 16, 1100, 256
+    rng = np.random.default_rng(3)
+    pages = (T + page - 1) // page
+    k = np.zeros((pages, 1, page, dim), np.float32)
+    k[..., 0] = -1.0
+    k[0, 0, 0, 0] = 1.0
+    v = rng.standard_normal((pages, 1, page, dim)).astype(np.float32)
+    q = np.zeros((T, 1, dim), np.float32)
+    q[..., 0] = 60.0  # scores +60 and -60 at scale 1
+    bits, up = hb.quant.bf16_bits, DeviceBuffer.from_array
+    qg = np.zeros((T, 1, 2 * dim), np.float32)  # gate 1/2
+    nwo = hb.attn_workspace_floats(1, 1, dim, T, 1, T, split)
+    wo, wml, out = DeviceBuffer(4 * nwo), DeviceBuffer(4 * nwo // dim * 2 + 256), DeviceBuffer(T * dim * 2)
+    print("case: prompt attention with a sink key", flush=True)
+    hb.paged_attention(up(bits(q)), up(bits(k)), up(np.ascontiguousarray(bits(v).transpose(0, 1, 3, 2))),
+                       up(np.arange(pages, dtype=np.int32)[None]), pages, up(np.array([0, T], np.int32)),
+                       up(np.array([T], np.int32)), up(np.zeros(T, np.int32)), up(bits(qg)), 2 * dim, 1, T, T, T, 1, 1,
+                       dim, 1.0, split, wo, wml, out)
+    hb.synchronize()
+    got = hb.quant.bf16_value(out.download(np.uint16, (T, dim)))
+    want = np.repeat(0.5 * hb.quant.bf16_value(bits(v))[0, 0, :1], T, 0)
+    assert_bf16_close(got, want, "sink")
