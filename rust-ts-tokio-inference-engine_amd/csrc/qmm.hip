@@ -16,6 +16,7 @@
 // 1 KB read and every scale/bias load a contiguous 128-byte read. All loads of
 // a wave are issued before its first MFMA; partial tiles are reduced in LDS.
 #include "qmm.h"
+#include "block_gemm.h"
 #include "proj_gemm.h"
 #include "proj_stream.h"
 #include "stream_gemm.h"
@@ -282,6 +283,19 @@ void qmm(const bf16_t* x, int M, int K, const uint32_t* w, const bf16_t* scales,
     // tiles of its block) for shapes outside the K-sliced family; otherwise the
     // streaming kernel, which reads the weights once for all tiles (the
     // per-tile kernel re-reads them)
+    {
+      bool block = false;
+      if (out_mode == 2)
+        block = block_gemm<2>(x, M, K, w, scales, N, y, ldy, stream);
+      else if (out_mode == 1)
+        block = block_gemm<1>(x, M, K, w, scales, N, y, ldy, stream);
+      else
+        block = block_gemm<0>(x, M, K, w, scales, N, y, ldy, stream);
+      if (block) {
+        HB_CHECK(hipGetLastError());
+        return;
+      }
+    }
     if (M > 16 && !dense_sliced(N, K)) {
       bool proj = false;
       if (gsum && reinterpret_cast<uintptr_t>(gsum) % 16) gsum = nullptr;  // loaded as uint4

@@ -157,3 +157,44 @@ def test_paged_attention_prompt_sink(hb):
     got = hb.quant.bf16_value(out.download(np.uint16, (T, dim)))
     want = np.repeat(0.5 * hb.quant.bf16_value(bits(v))[0, 0, :1], T, 0)
     assert_bf16_close(got, want, "sink")
+
+
+# one token more than the streamed projection takes, last blocks of 1, 33, 96 and
+# 65 tokens, K of a single group pair, of no whole number of 16 groups, and of the
+# output projections (fewer than 160 blocks stay with the older kernels, whose
+# codes' offset is 128 and whose bound is not this one)
+@pytest.mark.parametrize("M,N,K", [(257, 13824, 128), (321, 10240, 2048), (1920, 2048, 4096), (833, 4608, 1152)])
+def test_qmm_blocks(hb, M, N, K):
+    """The block form (more than 256 tokens, 160 blocks) in every output mode, rows wider than
+    N, against float64. f32 outputs: each of the K / 64 <= 64 group terms is
+    rounded at 2^-24 of a partial sum of at most some 16 times the output's rms
+    (the codes' offset of 16 against their spread of 4.6): 64 * 2^-24 * 4 = 1.5e-5
+    of the rms at the worst; bf16: 2^-8 of the value more."""
+    from hip_bridge import DeviceBuffer
+
+    rng = np.random.default_rng(M + K)
+    x, packed, s, b = hb.quant.qgemv_workload(M, N, K, seed=M + N)
+    tw = hb.TiledWeight(packed, s, b)
+    val = hb.quant.bf16_value
+    codes = ((packed[:, :, None] >> (4 * np.arange(8, dtype=np.uint32))) & 15).reshape(N, K).astype(np.float64)
+    w = codes * np.repeat(val(s).astype(np.float64), 64, 1) + np.repeat(val(b).astype(np.float64), 64, 1)
+    want = val(x).astype(np.float64) @ w.T
+    rms = np.sqrt(np.mean(want * want))
+    ldy = N + 32
+    init = rng.standard_normal((M, ldy)).astype(np.float32)
+    dx = DeviceBuffer.from_array(x)
+    for mode in (0, 1, 2):
+        print(f"case: block qmm {M}x{N}x{K} mode {mode}", flush=True)
+        dy = DeviceBuffer.from_array(init)
+        hb.qmm(dx, tw.w, tw.sb, None, dy, M, N, K, ldy=ldy, out_mode=mode)
+        hb.synchronize()
+        if mode == 0:
+            got = val(dy.download(np.uint16, (M, ldy)))[:, :N].astype(np.float64)
+            assert np.all(np.abs(got - want) <= 2.0**-8 * np.abs(want) + 1.5e-5 * rms), np.abs(got - want).max() / rms
+            continue
+        got = dy.download(np.float32, (M, ldy))
+        assert np.array_equal(got[:, N:], init[:, N:]), "columns past N untouched"
+        base = init[:, :N].astype(np.float64) if mode == 2 else 0.0
+        err = np.abs(got[:, :N] - (want + base)).max() / rms
+        print(f"  max error / rms {err:.2e}")
+        assert err < 1.5e-5
