@@ -522,7 +522,8 @@ Engine::Engine(const rs_qwen_config& cfg, int max_rows, int max_context, int max
   gb_ = falloc(size_t(Tm) * g.Hv);
   if (g.H % 64 == 0) hgs_ = falloc(size_t(Tm) * (g.H / 64));
   y_ = balloc(size_t(Tm) * g.Hv * g.Dv);
-  const int chunk = std::min(Tm, kMoeChunk);
+  moe_block_ = moe_block_fits(std::min(Tm, kMoeBlockTokens), g.E, g.top, g.H, g.I);
+  const int chunk = std::min(Tm, moe_block_ ? kMoeBlockTokens : kMoeChunk);
   rlog_ = falloc(size_t(chunk) * g.router_rows());
   moe_idx_ = ialloc(size_t(chunk) * g.top);
   moe_w_ = falloc(size_t(chunk) * g.top);
@@ -530,7 +531,8 @@ Engine::Engine(const rs_qwen_config& cfg, int max_rows, int max_context, int max
   moe_offsets_ = ialloc(g.E + 1);
   moe_order_ = ialloc(size_t(chunk) * g.top);
   moe_inverse_ = ialloc(size_t(chunk) * g.top);
-  moe_items_ = ialloc(moe_items_capacity(chunk, g.E, g.top));
+  moe_items_ = ialloc(std::max(moe_items_capacity(std::min(Tm, kMoeChunk), g.E, g.top),
+                               moe_block_ ? moe_block_items_capacity(chunk, g.E, g.top) : size_t(0)));
   act_ = balloc(size_t(chunk) * (g.top + 1) * g.I);
   dout_ = balloc(size_t(chunk) * (g.top + 1) * g.H);
   logits_ = falloc(size_t(Tm) * g.vocab_rows());
@@ -660,21 +662,27 @@ void Engine::moe_block(const LayerW& w, int T, const CombineNorm* next, bool cut
   if (cut_norm) op_begin();
   rmsnorm(x_, g.H, w.post_norm, T, g.H, g.eps, h_, g.H, stream_);
   if (cut_norm) op_cut(OpStage::ResidualNorm);
-  for (int c0 = 0; c0 < T; c0 += kMoeChunk) {
-    const int n = std::min(kMoeChunk, T - c0);
+  // prompts: chunks of up to 4096 tokens, whose experts' rows fill whole tiles
+  const bool blocks = moe_block_ && !w.g_gate_up.on() && !w.g_down.on();
+  for (int c0 = 0, n; c0 < T; c0 += n) {
+    const bool block = blocks && T - c0 > kMoeBlockMin;
+    n = std::min(block ? kMoeBlockTokens : kMoeChunk, T - c0);
     const bf16_t* hc = h_ + size_t(c0) * g.H;
     op_begin();
     project(w.router, w.g_router, hc, n, rlog_, 1, w.router.N);
     const bool sampled = probe_sample(0);
     int32_t* census = sampled && probe_[0].n < kProbeCap ? census_ + probe_[0].n : nullptr;
-    moe_route(rlog_, w.router.N, n, g.E, g.top, moe_idx_, moe_w_, moe_counts_, moe_offsets_, moe_order_,
-              moe_inverse_, moe_items_, stream_, census);
+    (block ? moe_route_block : moe_route)(rlog_, w.router.N, n, g.E, g.top, moe_idx_, moe_w_, moe_counts_,
+                                          moe_offsets_, moe_order_, moe_inverse_, moe_items_, stream_, census);
     op_cut(OpStage::MoeRouting);
     op_begin();
     probe_begin(0, sampled);
     if (w.g_gate_up.on()) {
       const auto& m = w.g_gate_up.mods;  // experts' gate, up, then the shared expert's
       moe_generic_gate_up(hc, g.H, moe_order_, moe_idx_, g.top, n * g.top, n, m[0], m[1], m[2], m[3], act_, stream_);
+    } else if (block) {
+      moe_block_qmm(hc, g.H, w.gate_up.w, w.gate_up.sb, 2 * g.I, moe_order_, moe_items_, g.E, g.top, n, 1, act_,
+                    stream_);
     } else {
       moe_grouped_qmm(hc, g.H, w.gate_up.w, w.gate_up.sb, 2 * g.I, moe_counts_, moe_offsets_, moe_order_,
                       moe_items_, g.E, g.top, n, 1, act_, stream_);
@@ -686,6 +694,8 @@ void Engine::moe_block(const LayerW& w, int T, const CombineNorm* next, bool cut
     if (w.g_down.on()) {
       const auto& m = w.g_down.mods;
       moe_generic_down(act_, moe_order_, moe_idx_, g.top, n * g.top, n, m[0], m[1], dout_, stream_);
+    } else if (block) {
+      moe_block_qmm(act_, g.I, w.down.w, w.down.sb, g.H, moe_order_, moe_items_, g.E, g.top, n, 0, dout_, stream_);
     } else {
       moe_grouped_qmm(act_, g.I, w.down.w, w.down.sb, g.H, moe_counts_, moe_offsets_, moe_order_, moe_items_, g.E,
                       g.top, n, 0, dout_, stream_);

@@ -365,6 +365,7 @@ class Engine {
   float* hgs_ = nullptr;  // per-64-column group sums of h_ from the norm that wrote it (null: hidden % 64 != 0)
   bf16_t *h_, *proj_, *q_, *aout_, *y_, *act_, *dout_, *hn_, *sel_h_;
   int32_t *moe_idx_, *moe_counts_, *moe_offsets_, *moe_order_, *moe_inverse_, *moe_items_, *sel_status_;
+  bool moe_block_ = false;  // prompt-sized chunks take the block form (moe_block_fits)
   uint32_t* winners_;
   void* sel_ws_ = nullptr;
   void* sel_part_ = nullptr;  // fused selection partials

@@ -55,6 +55,27 @@ void moe_combine(const bf16_t* down, const float* weights, const int32_t* invers
                  int ld_logits, int sg_col, int top, int tokens, int hidden, float* residual, hipStream_t stream,
                  const CombineNorm* norm = nullptr);
 
+// The same block for prompt-sized chunks (kMoeBlockMin < tokens <=
+// kMoeBlockTokens): the experts' pairs in tiles of up to 96 rows, each weight
+// matrix read once per tile. moe_route_block writes what moe_route does, except
+// that an expert's pairs are in no fixed order (no row's value depends on its
+// place) and items (moe_block_items_capacity int32) lists the tiles: items[0] =
+// count, then from 4 on one (expert, first output row, rows, 0) quadruple each,
+// the shared expert's first. moe_block_fits: the geometries both take.
+// Chunks of 256 tokens re-read every expert (512 of width 512, hidden 2048: 167
+// us of products and 28 us of routing each); one chunk of up to 4096 takes 285
+// us at 260 to 1,000 tokens and 490 us at 4,000, so it is the shorter from about
+// 290 tokens on.
+constexpr int kMoeBlockMin = 288, kMoeBlockTokens = 4096;
+bool moe_block_fits(int tokens, int experts, int top, int hidden, int intermediate);
+size_t moe_block_items_capacity(int tokens, int experts, int top);
+void moe_route_block(const float* logits, int ld_logits, int tokens, int experts, int top, int32_t* idx, float* weights,
+                     int32_t* counts, int32_t* offsets, int32_t* order, int32_t* inverse, int32_t* items,
+                     hipStream_t stream, int32_t* active = nullptr);
+void moe_block_qmm(const bf16_t* x, int K, const uint32_t* w_tiled, const bf16_t* sb_tiled, int n_rows,
+                   const int32_t* order, const int32_t* items, int experts, int top, int tokens, int swiglu,
+                   bf16_t* y, hipStream_t stream);
+
 // out[0] = number of experts with counts[e] > 0 (the routed experts whose
 // weights one grouped GEMM launch reads).
 void moe_count_active(const int32_t* counts, int experts, int32_t* out, hipStream_t stream);

@@ -19,6 +19,7 @@
 
 #include <type_traits>
 
+#include "block_gemm.h"
 #include "moe_gemm.h"
 #include "q4_device.h"
 
@@ -726,19 +727,9 @@ void launch_grouped(const bf16_t* x, int K, const uint32_t* w, const bf16_t* sb,
 
 }  // namespace
 
-size_t moe_items_capacity(int tokens, int experts, int top) {
-  return size_t(moe_records_offset(tokens, experts, top)) + 16 * size_t(moe_list_capacity(tokens, experts, top));
-}
-
-void moe_route(const float* logits, int ld_logits, int tokens, int experts, int top, int32_t* idx, float* weights,
-               int32_t* counts, int32_t* offsets, int32_t* order, int32_t* inverse, int32_t* items,
-               hipStream_t stream, int32_t* active) {
-  require(logits && idx && weights && counts && offsets && order && inverse && items, "moe_route: null pointer");
-  require(tokens <= 65535 * 16, "moe_route: too many tokens for the work-item encoding");
-  require(experts > 0 && experts <= kMaxExperts, "moe_route: experts must be 1..1024");
-  require(top > 0 && top <= experts && top <= 16, "moe_route: top must be 1..16 and <= experts");
-  require(tokens > 0 && tokens * top <= kMoeMaxPairs, "moe_route: tokens * top exceeds one routing workgroup");
-  require(ld_logits >= experts, "moe_route: logits row stride");
+namespace {
+void moe_topk(const float* logits, int ld_logits, int tokens, int experts, int top, int32_t* idx, float* weights,
+              hipStream_t stream) {
   const dim3 tg((tokens + kTopkWaves - 1) / kTopkWaves), tb(64 * kTopkWaves);
   const int per = (experts + 63) / 64;
   if (per <= 1)
@@ -752,6 +743,23 @@ void moe_route(const float* logits, int ld_logits, int tokens, int experts, int 
   else
     hipLaunchKernelGGL(moe_topk_kernel<16>, tg, tb, 0, stream, logits, ld_logits, tokens, experts, top, idx, weights);
   HB_CHECK(hipGetLastError());
+}
+}  // namespace
+
+size_t moe_items_capacity(int tokens, int experts, int top) {
+  return size_t(moe_records_offset(tokens, experts, top)) + 16 * size_t(moe_list_capacity(tokens, experts, top));
+}
+
+void moe_route(const float* logits, int ld_logits, int tokens, int experts, int top, int32_t* idx, float* weights,
+               int32_t* counts, int32_t* offsets, int32_t* order, int32_t* inverse, int32_t* items,
+               hipStream_t stream, int32_t* active) {
+  require(logits && idx && weights && counts && offsets && order && inverse && items, "moe_route: null pointer");
+  require(tokens <= 65535 * 16, "moe_route: too many tokens for the work-item encoding");
+  require(experts > 0 && experts <= kMaxExperts, "moe_route: experts must be 1..1024");
+  require(top > 0 && top <= experts && top <= 16, "moe_route: top must be 1..16 and <= experts");
+  require(tokens > 0 && tokens * top <= kMoeMaxPairs, "moe_route: tokens * top exceeds one routing workgroup");
+  require(ld_logits >= experts, "moe_route: logits row stride");
+  moe_topk(logits, ld_logits, tokens, experts, top, idx, weights, stream);
   const int words = experts * ((tokens + 63) / 64);
   if (words <= kBitmapWords)
     hipLaunchKernelGGL(moe_sort_bitmap_kernel, dim3(1), dim3(kSortThreads), size_t(words) * 8, stream, idx, tokens, top,
@@ -794,6 +802,200 @@ void moe_grouped_qmm(const bf16_t* x, int K, const uint32_t* w_tiled, const bf16
       launch_grouped<2, false>(x, K, w_tiled, sb_tiled, n_rows, counts, offsets, order, experts, top, tokens, y,
                                stream);
   }
+  HB_CHECK(hipGetLastError());
+}
+
+namespace {
+// Counting sort of the (token, slot) pairs of a prompt-sized chunk by expert and
+// the list of its tiles, one workgroup: counts and places with LDS atomics, so
+// the pairs of an expert are in no fixed order. One pass over up to 40,960 pairs
+// (33 us) where the 256-token chunks took a sort each (7 us, sixteen times for
+// 4,000 tokens).
+__global__ __launch_bounds__(kSortThreads) void moe_sort_block_kernel(const int32_t* __restrict__ idx, int T, int top,
+                                                                      int E, int32_t* __restrict__ counts,
+                                                                      int32_t* __restrict__ offsets,
+                                                                      int32_t* __restrict__ order,
+                                                                      int32_t* __restrict__ inverse,
+                                                                      int32_t* __restrict__ items,
+                                                                      int32_t* __restrict__ active) {
+  __shared__ int32_t cnt[kMaxExperts];
+  __shared__ int32_t scan[33];
+  const int P = T * top, tid = threadIdx.x;
+  constexpr int kAhead = 8;
+  for (int e = tid; e < kMaxExperts; e += kSortThreads) cnt[e] = 0;
+  __syncthreads();
+  for (int p0 = tid; p0 < P; p0 += kAhead * kSortThreads) {
+    int e[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) e[k] = idx[min(p0 + k * kSortThreads, P - 1)];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k)
+      if (p0 + k * kSortThreads < P) atomicAdd(&cnt[e[k]], 1);
+  }
+  __syncthreads();
+  const int v = tid < E ? cnt[tid] : 0;
+  int total;
+  const int excl = block_exclusive_scan(v, scan, &total);
+  const int shared_tiles = (T + kBgTok - 1) / kBgTok, tiles = (v + kBgTok - 1) / kBgTok;
+  int total_tiles;
+  const int first = shared_tiles + block_exclusive_scan(tiles, scan, &total_tiles);
+  int4* const list = reinterpret_cast<int4*>(items + 4);
+  for (int j = 0; j < tiles; ++j)
+    list[first + j] = make_int4(tid, excl + kBgTok * j, min(kBgTok, v - kBgTok * j), 0);
+  for (int j = tid; j < shared_tiles; j += kSortThreads)
+    list[j] = make_int4(E, P + kBgTok * j, min(kBgTok, T - kBgTok * j), 0);
+  if (tid == 0) items[0] = shared_tiles + total_tiles;
+  if (active) {
+    int n_active;
+    block_exclusive_scan(v > 0 ? 1 : 0, scan, &n_active);
+    if (tid == 0) active[0] = n_active;
+  }
+  if (tid < E) {
+    counts[tid] = v;
+    offsets[tid] = excl;
+    cnt[tid] = excl;
+  }
+  if (tid == E - 1) offsets[E] = excl + v;
+  __syncthreads();
+  for (int p0 = tid; p0 < P; p0 += kAhead * kSortThreads) {
+    int e[kAhead];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) e[k] = idx[min(p0 + k * kSortThreads, P - 1)];
+#pragma unroll
+    for (int k = 0; k < kAhead; ++k) {
+      const int p = p0 + k * kSortThreads;
+      if (p >= P) break;
+      const int dst = atomicAdd(&cnt[e[k]], 1);
+      order[dst] = p;
+      inverse[p] = dst;
+    }
+  }
+}
+
+// One tile's product with a block of 256 weight rows (block_gemm.h), with the
+// SwiGLU of the gate/up matrix in the epilogue: a 16-row tile holds 8 gate rows,
+// then their up rows, so gate lane n and up lane n ^ 8 exchange one of two
+// tokens and each finishes the other.
+template <bool SWIGLU, int TT>
+__device__ inline void moe_block_tile(const BgBlock& blk, const uint32_t (&xoff)[kBgTokWave / 8], int PK, uint4* lds,
+                                      bf16_t* __restrict__ y, int ldy, size_t m0, int row0) {
+  f32x16 total[TT][2];
+  bg_run<TT>(blk, xoff, PK, lds, total);
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6, n32 = lane & 31, h = lane >> 5;
+  const int up = (lane >> 3) & 1, odd = lane & 1;
+#pragma unroll
+  for (int t = 0; t < TT; ++t)
+#pragma unroll
+    for (int j = 0; j < 2; ++j)
+#pragma unroll
+      for (int r = 0; r < 16; r += 2) {
+        float a = total[t][j][r], b = total[t][j][r + 1];
+        asm("" : "+v"(a), "+v"(b));  // two registers to choose from, not an index into sixteen
+        const int m = 32 * t + 8 * (r >> 2) + 4 * h + (r & 3);
+        const int sel = SWIGLU ? up : odd;
+        const float give = sel ? a : b, keep = sel ? b : a;
+        if constexpr (SWIGLU) {
+          const float got = __builtin_bit_cast(
+              float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give), 0x128, 0xF, 0xF, false));
+          const float g = up ? got : keep, u = up ? keep : got;
+          const int col = (row0 + 64 * wave + 32 * j) / 2 + (n32 >> 4) * 8 + (lane & 7);
+          if (m + up < blk.rows) y[(m0 + m + up) * ldy + col] = f32_to_bf16(g / (1.f + __expf(-g)) * u);
+        } else {
+          const float got = __builtin_bit_cast(
+              float, __builtin_amdgcn_update_dpp(0, __builtin_bit_cast(int, give), 0xB1, 0xF, 0xF, false));
+          const uint32_t pair = odd ? bg_pack(got, keep) : bg_pack(keep, got);
+          const int col = row0 + 64 * wave + 32 * j + (n32 & ~1);
+          if (m + odd < blk.rows) *reinterpret_cast<uint32_t*>(y + (m0 + m + odd) * ldy + col) = pair;
+        }
+      }
+}
+
+// 4,000 tokens, top-10 of 512 experts of width 512: gate/up 308 us (0.60
+// PFLOP/s of the live rows), down 183 us, against 16 x 107 and 16 x 60 us of
+// 256-token chunks. At 260 to 1,000 tokens (175 + 101 us) the launch is the
+// stream of the experts' weights, 0.9 GB.
+// Block b on XCD b % 8: the row blocks of a tile follow each other on one XCD and
+// read its x rows from that XCD's L2; blocks past the list leave at once.
+template <bool SWIGLU>
+__global__ __launch_bounds__(kBgThreads, 2) void moe_block_kernel(const bf16_t* __restrict__ x, int PK,
+                                                                const uint32_t* __restrict__ wt,
+                                                                const bf16_t* __restrict__ sbt, int n_rows,
+                                                                const int32_t* __restrict__ order,
+                                                                const int32_t* __restrict__ items, int E, int top,
+                                                                int P, bf16_t* __restrict__ y, int ldy) {
+  extern __shared__ uint4 lds[];
+  const int rblocks = n_rows / kBgRows;
+  const int j8 = blockIdx.x / 8, rb = j8 % rblocks, item = (j8 / rblocks) * 8 + blockIdx.x % 8;
+  if (item >= items[0]) return;  // uniform over the workgroup
+  const int4 it = reinterpret_cast<const int4*>(items + 4)[item];
+  const int e = it.x, base = it.y, rows = it.z, K = PK * 128;
+  const size_t tile16 = (size_t(e) * rblocks + rb) * (kBgRows / 16);
+  BgBlock blk{SWIGLU ? x : x + size_t(base) * K, rows, reinterpret_cast<const uint4*>(wt) + tile16 * PK * 64,
+              reinterpret_cast<const uint2*>(sbt) + tile16 * PK * 16};
+  const int lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
+  uint32_t xoff[kBgTokWave / 8];
+#pragma unroll
+  for (int i = 0; i < kBgTokWave / 8; ++i) {
+    const int t = kBgTokWave * wave + 8 * i + (lane >> 3), m = min(t, rows - 1);
+    int src = m;
+    if (SWIGLU) src = e < E ? order[base + m] / top : base - P + m;
+    xoff[i] = uint32_t(src) * uint32_t(K) * 2u + ((lane & 7) ^ ((t >> 1) & 7)) * 16;
+  }
+  if (rows > 64)
+    moe_block_tile<SWIGLU, 3>(blk, xoff, PK, lds, y, ldy, base, rb * kBgRows);
+  else if (rows > 32)
+    moe_block_tile<SWIGLU, 2>(blk, xoff, PK, lds, y, ldy, base, rb * kBgRows);
+  else
+    moe_block_tile<SWIGLU, 1>(blk, xoff, PK, lds, y, ldy, base, rb * kBgRows);
+}
+
+int moe_block_tiles(int tokens, int experts, int top) {  // at most
+  return (tokens + kBgTok - 1) / kBgTok + std::min(experts, tokens * top) + tokens * top / kBgTok;
+}
+
+}  // namespace
+
+bool moe_block_fits(int tokens, int experts, int top, int hidden, int intermediate) {
+  return tokens > kMoeBlockMin && tokens <= kMoeBlockTokens && experts >= 1 && experts <= kMaxExperts && top >= 1 &&
+         top <= experts && top <= 16 && hidden % kBgRows == 0 && (2 * intermediate) % kBgRows == 0 &&
+         intermediate % 128 == 0 && int64_t(tokens) * hidden * 2 <= INT32_MAX;
+}
+
+size_t moe_block_items_capacity(int tokens, int experts, int top) {
+  return 4 + 4 * size_t(moe_block_tiles(tokens, experts, top));
+}
+
+void moe_route_block(const float* logits, int ld_logits, int tokens, int experts, int top, int32_t* idx, float* weights,
+                     int32_t* counts, int32_t* offsets, int32_t* order, int32_t* inverse, int32_t* items,
+                     hipStream_t stream, int32_t* active) {
+  require(logits && idx && weights && counts && offsets && order && inverse && items, "moe_route_block: null pointer");
+  require(tokens > 0 && tokens <= kMoeBlockTokens && experts > 0 && experts <= kMaxExperts && top > 0 &&
+              top <= experts && top <= 16 && ld_logits >= experts,
+          "moe_route_block: geometry");
+  moe_topk(logits, ld_logits, tokens, experts, top, idx, weights, stream);
+  hipLaunchKernelGGL(moe_sort_block_kernel, dim3(1), dim3(kSortThreads), 0, stream, idx, tokens, top, experts, counts,
+                     offsets, order, inverse, items, active);
+  HB_CHECK(hipGetLastError());
+}
+
+void moe_block_qmm(const bf16_t* x, int K, const uint32_t* w_tiled, const bf16_t* sb_tiled, int n_rows,
+                   const int32_t* order, const int32_t* items, int experts, int top, int tokens, int swiglu,
+                   bf16_t* y, hipStream_t stream) {
+  require(x && w_tiled && sb_tiled && order && items && y, "moe_block_qmm: null pointer");
+  require(n_rows % kBgRows == 0 && K % 128 == 0 && tokens > 0 && tokens <= kMoeBlockTokens &&
+              int64_t(tokens) * K * 2 <= INT32_MAX,
+          "moe_block_qmm: geometry");
+  const int rblocks = n_rows / kBgRows, tiles = moe_block_tiles(tokens, experts, top);
+  const auto kernel = swiglu ? moe_block_kernel<true> : moe_block_kernel<false>;
+  static const hipError_t attr[2] = {
+      hipFuncSetAttribute(reinterpret_cast<const void*>(moe_block_kernel<false>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, int(kBgLds)),
+      hipFuncSetAttribute(reinterpret_cast<const void*>(moe_block_kernel<true>),
+                          hipFuncAttributeMaxDynamicSharedMemorySize, int(kBgLds))};
+  HB_CHECK(attr[0]);
+  HB_CHECK(attr[1]);
+  launch_timed(kernel, dim3(unsigned((tiles + 7) / 8 * 8) * rblocks), dim3(kBgThreads), kBgLds, stream, x, K / 128,
+               w_tiled, sb_tiled, n_rows, order, items, experts, top, tokens * top, y, swiglu ? n_rows / 2 : n_rows);
   HB_CHECK(hipGetLastError());
 }
 

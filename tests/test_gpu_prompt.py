@@ -198,3 +198,70 @@ def test_qmm_blocks(hb, M, N, K):
         err = np.abs(got[:, :N] - (want + base)).max() / rms
         print(f"  max error / rms {err:.2e}")
         assert err < 1.5e-5
+
+
+# 301 tokens: about 75, 38 and 9 rows per expert (tiles of three, two and one
+# 32-row products), a shared expert of three full tiles and one of 13 rows
+@pytest.mark.parametrize("experts", [8, 16, 64])
+def test_engine_prompt_matches_oracle(bridge, experts):
+    """A prompt step past the streaming kernels' 256 tokens, layer by layer
+    against the oracle: the MoE block form beside prompt attention and the
+    chunked recurrence, then one decode step on the state it left."""
+    from hip_bridge.engine import Engine, tiny_config
+    from layer_check import Row, check_layers
+    from oracle.model import HybridModel
+
+    cfg = tiny_config(layers=2, interval=2, experts=experts)
+    e = Engine(cfg, 2, 512, 260, 301, seed=experts, mtp=False)
+    try:
+        e.trace(True)
+        model = HybridModel(cfg.dims(), e.export)
+        model.tie_window = 2e-3
+        rng = np.random.default_rng(experts)
+        seqs = [rng.integers(0, cfg.vocab, n).astype(np.uint32) for n in (260, 41)]
+        print(f"case: engine prompt of 301 tokens, {experts} experts", flush=True)
+        e.forward([260, 41], [0, 0], [0, 1], np.concatenate(seqs), logit_rows=[259, 300])
+        trace, mid, logits = e.read("trace", 301), e.read("mid_trace", 301), e.read("logits", 2)
+        rows = []
+        for r, (a, b) in enumerate(((0, 260), (260, 301))):
+            row = Row(cfg.layers, cfg.hidden)
+            row.extend(trace[:, a:b], mid[:, a:b])
+            check_layers(model, row, b - a, seqs[r], f"row {r}")
+            assert_bf16_close(logits[r], model.head(row.x[cfg.layers][-1:])[1][0], f"logits row {r}")
+            rows.append(row)
+        nxt = rng.integers(0, cfg.vocab, 2).astype(np.uint32)
+        e.forward([1, 1], [260, 41], [0, 1], nxt, hist_off=[260, 41], logit_rows=[0, 1])
+        trace, mid = e.read("trace", 2), e.read("mid_trace", 2)
+        for r in range(2):
+            rows[r].extend(trace[:, r:r + 1], mid[:, r:r + 1])
+            check_layers(model, rows[r], 1, np.append(seqs[r], nxt[r]), f"decode after row {r}")
+    finally:
+        e.close()
+
+
+@pytest.mark.parametrize("last", [40, 304])
+def test_engine_step_of_two_moe_chunks(bridge, last):
+    """More tokens than one MoE chunk takes (4096), the rest in the decode form or
+    the block form: every row as in a step of its own. A token whose routing is
+    nearly tied may go to another expert there; 1 in 100 is allowed for."""
+    from hip_bridge.engine import Engine, tiny_config
+
+    cfg = tiny_config(layers=1, interval=2, context=2048)
+    lens = [1400, 1400, 1296 - 8, last + 8]
+    e = Engine(cfg, 4, 2048, 1400, sum(lens), seed=5, mtp=False)
+    try:
+        rng = np.random.default_rng(last)
+        seqs = [rng.integers(0, cfg.vocab, n).astype(np.uint32) for n in lens]
+        print(f"case: engine step of {sum(lens)} tokens", flush=True)
+        e.forward(lens, [0] * 4, [0, 1, 2, 3], np.concatenate(seqs))
+        got = e.read("hidden", sum(lens)).copy()
+        at = 0
+        for r, s in enumerate(seqs):
+            e.forward([len(s)], [0], [r], s)
+            want = e.read("hidden", len(s))
+            rms = np.sqrt(np.mean(want * want))
+            off = (np.abs(got[at:at + len(s)] - want).max(1) > 2e-2 * (np.abs(want).max(1) + rms)).mean()
+            assert off <= 0.01, f"row {r}: {off:.3f} of the tokens differ"
+            at += len(s)
+    finally:
+        e.close()
