@@ -56,11 +56,11 @@ struct AttnWork {
 // on the row alone.
 //
 // A lone row's q tiles are all that run beside each other, each walking the
-// row's keys at 34 ns a key, while the split kernel spreads them over the chip:
+// row's keys at 36 ns a key, while the split kernel spreads them over the chip:
 // 0.095 ns per token and key, plus some 15 us more for its list and merge.
 // So few tokens over many keys stay with the split (us, split / one launch: 64
 // tokens over 564 keys 28 / 31, over 964 29 / 44; 200 over 2,200 76 / 82; 256
-// over 6,256 177 / 213; 500 over 5,500 293 / 189; 500 over 500 83 / 30).
+// over 6,256 177 / 213; 500 over 5,500 293 / 202; 500 over 500 84 / 31).
 constexpr int kPrefillRowTokens = 64;
 template <class I>
 __host__ __device__ inline bool attn_prefill_row(I tokens, I context, int from) {

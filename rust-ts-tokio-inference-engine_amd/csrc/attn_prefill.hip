@@ -9,20 +9,20 @@
 // K and V are read once per 16 tokens and the result needs no merge: softmax,
 // division and the sigmoid gate end in the same kernel.
 //
-// Two groups of four waves take the row's 32-key tiles in turn. Wave w of a
+// Two groups of four waves take the row's 256-key chunks in turn. Wave w of a
 // group holds the q of pairs 32 w .. 32 w + 31 (64 registers) and their f32
 // output tile (256 dims x 32 pairs, 128 registers); 16 KB of K and of V go from
 // memory to LDS directly, one tile ahead, into two buffers per group. So a SIMD
 // runs one group's softmax beside the other's products, also where a short
-// prompt gives a CU only one workgroup (1,000 keys: 44 us a workgroup, 58 us
-// with one group), and the groups' halves meet once at the end. Scores are
+// prompt gives a CU only one workgroup (36 ns a key, 48 with one group), and
+// the groups' halves meet once at the end. Scores are
 // computed transposed, S^T = K . Q^T (v_mfma_f32_32x32x16_bf16), with the LDS
 // rows of K in the order that leaves a lane with the scores of keys
 // 8 h .. 8 h + 7 and 16 + 8 h .. 16 + 8 h + 7 of one pair (h its half of the
 // wave): the B operand of O^T += V^T . P^T as it stands.
 //
-// Three prompts of 1,500 tokens (129 GFLOP with the causal half left out): 1180
-// us as splits, 170 - 195 us here (0.7 PFLOP/s). What bounds it is LDS beside
+// Three prompts of 1,500 tokens (129 GFLOP with the causal half left out): 1215
+// us as splits, 213 us here (0.6 PFLOP/s). What bounds it is LDS beside
 // the registers: a 32-pair wave reads a tile's 32 KB for 1,024 cycles of MFMA,
 // which for four SIMDs is the LDS rate; a wave of 64 pairs would halve that and
 // does not fit the registers of two waves per SIMD, and with 254 of 256 in use
@@ -38,7 +38,8 @@ constexpr int kD = 256;       // head_dim
 constexpr int kTile = 32;     // keys per tile
 constexpr int kWaves = 4;            // waves of a key group
 constexpr int kPairs = 32 * kWaves;  // (token, q head) pairs per workgroup
-constexpr int kGroups = 2;           // key groups: group g takes tiles g, g + 2, ...
+constexpr int kGroups = 2;           // key groups: group g takes 256-key chunks g, g + 2, ...
+constexpr int kChunk = 8;            // tiles of a chunk
 constexpr int kMatU4 = kTile * kD / 8;  // 16-byte units of a tile of K or of V
 constexpr int kBufU4 = 2 * kMatU4;
 constexpr int kBufs = 2;                // per key group
@@ -46,8 +47,6 @@ constexpr int kMergeU4 = kGroups * kWaves * 16 * 64;  // half of every wave's ou
 constexpr size_t kLds = size_t(kGroups) * kBufs * kBufU4 * 16 + kGroups * kWaves * 64 * 8;
 static_assert(kMergeU4 <= kGroups * kBufs * kBufU4, "the merge fits the key buffers");
 static_assert(kTile == 2 * kPage, "a tile is two pages");
-
-constexpr int kFresh = 4;  // tiles of a key group after which its running max starts afresh
 
 typedef float f32x2 __attribute__((ext_vector_type(2)));
 
@@ -126,13 +125,13 @@ __global__ __launch_bounds__(64 * kWaves * kGroups) void attn_prefill_kernel(
     const size_t block = (size_t(bt[min(2 * i + my_page, last_page)]) * Hkv + kh) * size_t(kPage * kD);
     const bf16_t* const kp = kcache + block;
     const bf16_t* const vp = vcache + block;
-    uint4* const kb = lds + (kg * kBufs + (i / kGroups & 1)) * kBufU4 + wave * 256;
+    uint4* const kb = lds + (kg * kBufs + (i & 1)) * kBufU4 + wave * 256;
 #pragma unroll
     for (int j = 0; j < 4; ++j) to_lds(kp + k_src[j], kb + j * 64);
 #pragma unroll
     for (int j = 0; j < 4; ++j) to_lds(vp + v_src[j], kb + kMatU4 + j * 64);
   };
-  if (kg < n_tiles) load_tile(kg);
+  if (kg * kChunk < n_tiles) load_tile(kg * kChunk);
 
   bf16x8 qf[16];  // B operand: dims 16 s + 8 h .. + 7 of this lane's pair
   {
@@ -150,17 +149,21 @@ __global__ __launch_bounds__(64 * kWaves * kGroups) void attn_prefill_kernel(
 
   const int row_u4 = n32 * 32, row_x = n32 & 15;
   const int v_u4 = n32 * 2 + (h ^ ((n32 >> 2) & 1) ^ ((n32 >> 3) & 1));
-  for (int i = kg; i - kg < n_tiles; i += kGroups) {  // both groups go round equally often
+  // both groups go round equally often, group 1 past the last tile if need be
+  int i = kg * kChunk;
+  auto after = [](int t) { return t % kChunk == kChunk - 1 ? t + 1 + (kGroups - 1) * kChunk : t + 1; };
+  for (int first = 0; first < n_tiles; first = after(first), i = after(i)) {
     // this wave's share of tile i is in LDS, then everyone's; and every wave is
     // done with the buffer the next tile goes to
     __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0)
     __builtin_amdgcn_fence(__ATOMIC_RELEASE, "workgroup", "local");
     __builtin_amdgcn_s_barrier();
     __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "workgroup", "local");
-    if (i + kGroups < n_tiles) load_tile(i + kGroups);
+    const int next = after(i);
+    if (next < n_tiles) load_tile(next);
     const int j0 = i * kTile;
     if (i >= n_tiles || j0 > pos_max) continue;  // uniform over the wave; the barriers are at the top
-    const uint4* const kb = lds + (kg * kBufs + (i / kGroups & 1)) * kBufU4;
+    const uint4* const kb = lds + (kg * kBufs + (i & 1)) * kBufU4;
     const uint4* const vb = kb + kMatU4;
     f32x16 s;
 #pragma unroll
@@ -190,7 +193,7 @@ __global__ __launch_bounds__(64 * kWaves * kGroups) void attn_prefill_kernel(
     // for 4 % of the time, which is what the extra rescales cost. It stays
     // within 2^16 of the row's max, so what earlier keys left cannot overflow
     // (256 keys below that weigh less than 0.4 % together).
-    const bool fresh = i / kGroups % kFresh == 0;
+    const bool fresh = i % kChunk == 0;
     if (__builtin_amdgcn_ballot_w64(mx > m) || fresh) {
       row_max = fmaxf(row_max, mx);
       const float m_new = fresh ? fmaxf(mx, row_max - 16.f) : fmaxf(m, mx);
