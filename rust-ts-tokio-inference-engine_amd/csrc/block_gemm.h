@@ -102,6 +102,15 @@ __device__ inline float bg_unit_sum(u32x4 v) {
   return __builtin_amdgcn_fdot2_f32_bf16(__builtin_bit_cast(b2, uint32_t(v[3])), one, s, false);
 }
 
+// Workgroup barrier for LDS, without the fences at which the compiler waits for
+// every load to LDS under way: this wave's own LDS operations are done, and the
+// compiler moves none across
+__device__ inline void bg_barrier() {
+  asm volatile("" ::: "memory");
+  __builtin_amdgcn_s_waitcnt(0xc07f);  // lgkmcnt(0)
+  __builtin_amdgcn_s_barrier();
+  asm volatile("" ::: "memory");
+}
 // Keeps this wave's LDS reads behind its own loads to LDS (waited for before it)
 __device__ inline void wave_lds_order() { __builtin_amdgcn_fence(__ATOMIC_SEQ_CST, "wavefront", "local"); }
 
@@ -141,7 +150,15 @@ __device__ inline void bg_run(const BgBlock& blk, const uint32_t (&xoff)[kBgTokW
   const int wread = (n32 >> 4) * 64 + 32 * h + (lane & 15);
   const uint2* const sp = blk.sb + size_t(4 * wave + (n32 >> 4)) * PK * 16 + (lane & 15);
   uint2 sbr[2];
-  float sc1[2];  // scales of a pair's second group
+  float psc[2][2];  // [group of the pair][32-row tile] scales
+  auto scales = [&] {
+#pragma unroll
+    for (int j = 0; j < 2; ++j) {
+      psc[0][j] = __builtin_bit_cast(float, sbr[j].x << 16);
+      psc[1][j] = __builtin_bit_cast(float, sbr[j].y << 16);
+      asm volatile("" : "+v"(psc[0][j]), "+v"(psc[1][j]));  // here, before newer loads are out
+    }
+  };
   auto load_w = [&](int p) {
     const int pc = min(p, PK - 1);
 #pragma unroll
@@ -187,6 +204,7 @@ __device__ inline void bg_run(const BgBlock& blk, const uint32_t (&xoff)[kBgTokW
     wave_lds_order();
     read_words(0, 0, v);
     dequant(v, 0, wf[0]);
+    scales();
   }
 
   int slot = 0;
@@ -203,22 +221,10 @@ __device__ inline void bg_run(const BgBlock& blk, const uint32_t (&xoff)[kBgTokW
         __builtin_amdgcn_s_waitcnt(0x0f73);  // vmcnt(3)
       else
         __builtin_amdgcn_s_waitcnt(0x0f77);  // vmcnt(7)
-      lds_barrier();
-      float sc[2];
-#pragma unroll
-      for (int j = 0; j < 2; ++j) {
-        if (gi == 0) {
-          sc[j] = __builtin_bit_cast(float, sbr[j].x << 16);
-          sc1[j] = __builtin_bit_cast(float, sbr[j].y << 16);
-        } else {
-          sc[j] = sc1[j];
-        }
-      }
-      if (gi == 0) {
-        __builtin_amdgcn_sched_barrier(0);  // the scales are read before newer loads are out
-        load_w(p + 1);
-        __builtin_amdgcn_sched_barrier(0);
-      }
+      bg_barrier();
+      const float sc[2] = {psc[gi][0], psc[gi][1]};
+      if (gi == 0) load_w(p + 1);
+      __builtin_amdgcn_sched_barrier(0);
       load_x(g + 2, slot == 0 ? 2 : slot - 1);
       const uint4* const xb = lds + slot * kBgStageU4;
       slot = slot == 2 ? 0 : slot + 1;
@@ -305,6 +311,7 @@ __device__ inline void bg_run(const BgBlock& blk, const uint32_t (&xoff)[kBgTokW
         }
       }
       scale(TT - 1, 1);
+      if (gi == 1) scales();
     }
     // the bias products of the last groups (a multiple of 16, or the rest of K)
     if ((2 * p + 2) % kBgSumGroups == 0 || p == PK - 1) {
@@ -325,7 +332,7 @@ __device__ inline void bg_run(const BgBlock& blk, const uint32_t (&xoff)[kBgTokW
         bb[j] = __builtin_bit_cast(bf16x8, vb);
         bs[j] = __builtin_bit_cast(bf16x8, vs);
       }
-      lds_barrier();  // every token's sums are written; the next stage's barrier ends their reading
+      bg_barrier();  // every token's sums are written; the next stage's barrier ends their reading
 #pragma unroll
       for (int t = 0; t < TT; ++t) {
         float f[8];
@@ -350,6 +357,7 @@ __device__ inline void bg_run(const BgBlock& blk, const uint32_t (&xoff)[kBgTokW
       }
     }
   }
+  __builtin_amdgcn_s_waitcnt(0x0f70);  // vmcnt(0): the repeated last loads may not outlive the workgroup's LDS
 }
 
 // two floats to a bf16 pair, round to nearest even
