@@ -388,7 +388,7 @@ int hb_moe_combine(const void* down, const float* weights, const int32_t* invers
 int hb_argmax_margin(const float* logits, int ld, int rows, int vocab, uint32_t* winner, float* margin,
                      int32_t* status, void* workspace, void* stream, char* error, size_t capacity);
 /* Optional workspace of hb_argmax_margin (device, bytes): with it, long rows
- * are scanned by several workgroups and merged in column order. */
+ * are scanned by several workgroups whose summaries are then merged. */
 size_t hb_argmax_workspace_bytes(int rows, int vocab);
 /* No counterpart in the reference. hb_argmax_margin with its multi-workgroup
  * scan, for callers that cannot allocate device memory (code under HIP graph

@@ -47,51 +47,84 @@ __global__ __launch_bounds__(kSelThreads) void argmax_margin_kernel(const float*
 
 // Two-level variant for long rows: grid (chunks, rows), each workgroup scans
 // kSelChunk columns and leaves its (best, second, non-finite) in part[row][chunk];
-// one thread per row then merges the chunks in column order.
+// one wave per row then merges the chunks.
 constexpr int kSelChunk = 8192;
 
-__global__ __launch_bounds__(kSelThreads) void argmax_partial_kernel(const float* __restrict__ logits, int ld,
-                                                                     int vocab, int nchunk,
-                                                                     uint4* __restrict__ part) {
-  const int chunk = blockIdx.x, r = blockIdx.y, tid = threadIdx.x;
-  const float* row = logits + size_t(r) * ld;
-  const int c0 = chunk * kSelChunk, c1 = min(vocab, c0 + kSelChunk);
-  Top2 t{0u, 0xFFFFFFFFu, 0u, false};
-  int bad = 0;
-  for (int i = c0 + tid; i < c1; i += kSelThreads) {
-    const float v = row[i];
-    if (!isfinite(v)) bad = 1;
-    t = merge(t, Top2{total_key(v), uint32_t(i), 0u, false});
-  }
-  __shared__ Top2 sp[kSelThreads];
-  __shared__ int sb[kSelThreads];
-  sp[tid] = t;
-  sb[tid] = bad;
-  __syncthreads();
-  for (int s = kSelThreads / 2; s > 0; s >>= 1) {
-    if (tid < s) {
-      sp[tid] = merge(sp[tid], sp[tid + s]);
-      sb[tid] |= sb[tid + s];
-    }
-    __syncthreads();
-  }
-  if (tid == 0) part[size_t(r) * nchunk + chunk] = make_uint4(sp[0].k1, sp[0].i1, sp[0].k2, (sp[0].has2 ? 1u : 0u) | (sb[0] ? 2u : 0u));
+// Merge over the wave's lanes (any order: the larger key wins, on equal keys the
+// lower index), every lane ending with the result.
+__device__ inline Top2 wave_merge(Top2 t) {
+#pragma unroll
+  for (int off = 1; off < 64; off <<= 1)
+    t = merge(t, Top2{uint32_t(__shfl_xor(int(t.k1), off, 64)), uint32_t(__shfl_xor(int(t.i1), off, 64)),
+                      uint32_t(__shfl_xor(int(t.k2), off, 64)), __shfl_xor(int(t.has2), off, 64) != 0});
+  return t;
 }
 
-__global__ void argmax_final_kernel(const uint4* __restrict__ part, int nchunk, int rows, uint32_t* __restrict__ winner,
-                                    float* __restrict__ margin, int32_t* __restrict__ status) {
-  const int r = blockIdx.x * blockDim.x + threadIdx.x;
-  if (r >= rows) return;
+// 1,024 threads, eight columns each, all loaded before the first is looked at:
+// with 256 threads walking 32 columns a single row's 19 workgroups took 15.8
+// us, here 5.1 (vocabulary 151,936; with the merge 20.3 and 8.7 us).
+constexpr int kPartThreads = 1024;
+constexpr int kPartPer = kSelChunk / kPartThreads;
+
+__global__ __launch_bounds__(kPartThreads) void argmax_partial_kernel(const float* __restrict__ logits, int ld,
+                                                                      int vocab, int nchunk,
+                                                                      uint4* __restrict__ part) {
+  const int chunk = blockIdx.x, r = blockIdx.y, tid = threadIdx.x;
+  const float* row = logits + size_t(r) * ld;
+  const int c0 = chunk * kSelChunk;
+  float v[kPartPer];
+#pragma unroll
+  for (int k = 0; k < kPartPer; ++k) v[k] = row[min(c0 + tid + k * kPartThreads, vocab - 1)];
   Top2 t{0u, 0xFFFFFFFFu, 0u, false};
   int bad = 0;
-  for (int c = 0; c < nchunk; ++c) {
+#pragma unroll
+  for (int k = 0; k < kPartPer; ++k) {
+    const int i = c0 + tid + k * kPartThreads;
+    if (i >= vocab) break;
+    if (!isfinite(v[k])) bad = 1;
+    t = merge(t, Top2{total_key(v[k]), uint32_t(i), 0u, false});
+  }
+  t = wave_merge(t);
+  const bool any_bad = __any(bad);
+  __shared__ Top2 sp[kPartThreads / 64];
+  __shared__ int sb[kPartThreads / 64];
+  if ((tid & 63) == 0) {
+    sp[tid >> 6] = t;
+    sb[tid >> 6] = any_bad;
+  }
+  __syncthreads();
+  if (tid >= 64) return;
+  const int w = tid & (kPartThreads / 64 - 1);
+  // lanes 16 further hold the same 16 summaries: merged over the 16 only
+  t = sp[w];
+  int b = sb[w];
+#pragma unroll
+  for (int off = 1; off < kPartThreads / 64; off <<= 1) {
+    t = merge(t, Top2{uint32_t(__shfl_xor(int(t.k1), off, 64)), uint32_t(__shfl_xor(int(t.i1), off, 64)),
+                      uint32_t(__shfl_xor(int(t.k2), off, 64)), __shfl_xor(int(t.has2), off, 64) != 0});
+    b |= __shfl_xor(b, off, 64);
+  }
+  if (tid == 0) part[size_t(r) * nchunk + chunk] = make_uint4(t.k1, t.i1, t.k2, (t.has2 ? 1u : 0u) | (b ? 2u : 0u));
+}
+
+// one wave per row: its chunks, 64 at a time
+__global__ __launch_bounds__(64) void argmax_final_kernel(const uint4* __restrict__ part, int nchunk,
+                                                          uint32_t* __restrict__ winner, float* __restrict__ margin,
+                                                          int32_t* __restrict__ status) {
+  const int r = blockIdx.x, lane = threadIdx.x;
+  Top2 t{0u, 0xFFFFFFFFu, 0u, false};
+  int bad = 0;
+  for (int c = lane; c < nchunk; c += 64) {
     const uint4 p = part[size_t(r) * nchunk + c];
     t = merge(t, Top2{p.x, p.y, p.z, (p.w & 1u) != 0});
     bad |= (p.w & 2u) != 0;
   }
+  t = wave_merge(t);
+  const bool any_bad = __any(bad);
+  if (lane) return;
   winner[r] = t.i1;
   margin[r] = t.has2 ? key_value(t.k1) - key_value(t.k2) : INFINITY;
-  status[r] = bad;
+  status[r] = any_bad;
 }
 
 __global__ void mtp_plan_kernel(const uint32_t* __restrict__ draft, const int32_t* __restrict__ n_draft,
@@ -183,11 +216,11 @@ void argmax_margin(const float* logits, int ld, int rows, int vocab, uint32_t* w
   if (rows <= 0) return;
   const int nchunk = (vocab + kSelChunk - 1) / kSelChunk;
   if (workspace && nchunk > 1) {
-    hipLaunchKernelGGL(argmax_partial_kernel, dim3(nchunk, rows), dim3(kSelThreads), 0, stream, logits, ld, vocab,
+    hipLaunchKernelGGL(argmax_partial_kernel, dim3(nchunk, rows), dim3(kPartThreads), 0, stream, logits, ld, vocab,
                        nchunk, static_cast<uint4*>(workspace));
     HB_CHECK(hipGetLastError());
-    hipLaunchKernelGGL(argmax_final_kernel, dim3((rows + 63) / 64), dim3(64), 0, stream,
-                       static_cast<const uint4*>(workspace), nchunk, rows, winner, margin, status);
+    hipLaunchKernelGGL(argmax_final_kernel, dim3(rows), dim3(64), 0, stream,
+                       static_cast<const uint4*>(workspace), nchunk, winner, margin, status);
     HB_CHECK(hipGetLastError());
     return;
   }

@@ -265,3 +265,36 @@ def test_engine_step_of_two_moe_chunks(bridge, last):
             at += len(s)
     finally:
         e.close()
+
+
+@pytest.mark.parametrize("vocab", [8193, 16384, 64 * 8192 + 1, 151936])
+def test_argmax_chunk_edges(hb, vocab):
+    """The two-level selection at its chunk edges: winner and runner-up on either
+    side of one, ties across waves and chunks, a row of equal values, a row of
+    -inf, a NaN, and more chunks than a wave has lanes."""
+    from hip_bridge import DeviceBuffer
+
+    rng = np.random.default_rng(vocab)
+    rows, ld = 7, vocab + 3
+    x = rng.standard_normal((rows, ld)).astype(np.float32)
+    x[0, 8191], x[0, 8192] = 9.0, 8.5
+    x[1, vocab - 1] = x[1, 63] = x[1, 64] = 9.0
+    x[2] = 1.25
+    x[3] = -np.inf
+    x[4, vocab - 1] = np.nan
+    x[5, 0], x[5, vocab - 1] = 7.5, 9.0
+    x[:, vocab:] = 1e30  # past the vocabulary
+    dx = DeviceBuffer.from_array(x)
+    ws = DeviceBuffer(int(hb.load().hb_argmax_workspace_bytes(rows, vocab)))
+    w, m, s = (DeviceBuffer(4 * rows) for _ in range(3))
+    print(f"case: argmax vocab {vocab}", flush=True)
+    hb.call("hb_argmax_margin", dx, ld, rows, vocab, w, m, s, ws, None)
+    hb.synchronize()
+    win, margin, status = w.download(np.uint32, rows), m.download(np.float32, rows), s.download(np.int32, rows)
+    for r in range(rows):
+        # total order: NaN above all; equal values, -inf among them, by the lower index
+        best = int(np.argmax(x[r, :vocab])) if r not in (3, 4) else {3: 0, 4: vocab - 1}[r]
+        want = best, np.nan if r in (3, 4) else x[r, best] - np.delete(x[r, :vocab], best).max()
+        assert win[r] == want[0], (r, win[r], want)
+        assert margin[r] == want[1] or (np.isnan(margin[r]) and np.isnan(want[1])), (r, margin[r], want)
+        assert bool(status[r]) == (not np.all(np.isfinite(x[r, :vocab]))), r
