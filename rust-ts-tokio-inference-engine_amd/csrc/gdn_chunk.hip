@@ -20,8 +20,8 @@
 //
 // One workgroup of 8 waves owns one (row, head), two waves per SIMD. Wave w
 // keeps the state rows of keys [16 w, 16 w + 16) in registers across the
-// row's chunks; in the token-parallel phases it works on token block w & 3
-// and value half w >> 2; in the block substitution it owns value columns
+// row's chunks; in the token-parallel phases it works on one token block and
+// value half w >> 2; in the block substitution it owns value columns
 // [16 w, 16 w + 16) for all 64 tokens, with the corrected values held in
 // registers (the 16x16x16 MFMA's output layout is its B-operand layout, so
 // U_j feeds the next block's product directly).
@@ -181,7 +181,10 @@ __global__ __launch_bounds__(kThreads, 1) void gdn_chunk_kernel(
   float* const fP = fA + 1024 * 4;                            // P [t][i] (swizzled chunks)
   const int h = blockIdx.x, r = blockIdx.y, lane = threadIdx.x & 63;
   const int w = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
-  const int tb = w & 3, hf = w >> 2;  // token block and value half of the token-parallel phases
+  // token block and value half of the token-parallel phases. Waves w and w + 4
+  // share a SIMD and the triangular products grow with the block, so a SIMD gets
+  // one early and one late block
+  const int tb = w < 4 ? w : 7 - w, hf = w >> 2;
   const int Hv = g.value_heads, Hk = g.key_heads, kh = h / (Hv / Hk);
   const int t0 = cu_seqlens[r], T = cu_seqlens[r + 1] - t0;
   if (T <= 0) return;  // uniform over the workgroup
@@ -374,6 +377,9 @@ __global__ __launch_bounds__(kThreads, 1) void gdn_chunk_kernel(
     }
 #pragma unroll
     for (int ci = 0; ci < 4; ++ci) {
+      // of the blocks past the diagonal only the next one of P is read (as zeros,
+      // in the 32-token step it shares with the diagonal's)
+      if (ci > tb + hf) continue;  // uniform over the wave
       const int i = 16 * ci + r16;
       const float Li = sL[i];
 #pragma unroll
