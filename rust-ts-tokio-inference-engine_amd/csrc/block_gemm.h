@@ -447,7 +447,8 @@ constexpr int kBgMinTokens = 256, kBgMinBlocks = 160;
 template <int OUT>
 bool block_gemm(const bf16_t* x, int M, int K, const uint32_t* w, const bf16_t* sb, int n_rows, void* y, int ldy,
                 hipStream_t stream) {
-  if (M <= kBgMinTokens || n_rows % kBgRows || K % 128) return false;
+  // a longer K is taken, or refused, by the other forms alone
+  if (M <= kBgMinTokens || n_rows % kBgRows || K % 128 || K > 4096) return false;
   if (OUT == 0 && (ldy % 2 || reinterpret_cast<uintptr_t>(y) % 4)) return false;
   const int rblocks = n_rows / kBgRows, tblocks = (M + kBgTok - 1) / kBgTok;
   const int64_t blocks = int64_t((rblocks + 7) / 8 * 8) * tblocks;
